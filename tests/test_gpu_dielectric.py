@@ -125,6 +125,50 @@ def test_general_inverse_nearly_dependent_columns(ctx, nb):
     dA.free()
 
 
+def _eliminate(a):
+    """In-place Gauss-Jordan inverse of an HPD matrix, one pivot at a time, in float64."""
+    a = a.copy()
+    for p in range(len(a)):
+        r, f = a[p] * (1 / a[p, p].real), a[:, p].copy()
+        b = a - np.outer(f, r)
+        b[p], b[:, p] = r, -f * (1 / a[p, p].real)
+        b[p, p] = 1 / a[p, p].real
+        a = b
+    return a
+
+
+@pytest.mark.parametrize("cond", [1e3, 1e6])
+@pytest.mark.parametrize("nb", [17, 20, 40, 42, 57, 64])
+def test_hpd_inverse_keeps_the_eliminations_accuracy(ctx, nb, cond):
+    """eps = 1 + V B B^H V with a dense v^1/2 of condition 1e3: the leading 16 x 16 blocks are as
+    ill conditioned as the matrix.  The blocked inverse performs the operations of the elimination
+    pivot by pivot, rounded in another association, so its error (geometric mean over eight
+    matrices, against extended precision) is of the same size; 2 is asked for.  Products with
+    explicit inverses of the 16 x 16 blocks reach 7 to 7000."""
+    g = np.random.default_rng(nb)
+    cn = lambda *s: g.standard_normal(s) + 1j * g.standard_normal(s)
+    A = []
+    for _ in range(8):
+        q = np.linalg.qr(cn(nb, nb))[0]
+        e = (q * np.logspace(0, -3, nb)) @ q.conj().T @ cn(nb, nb)
+        e = e @ e.conj().T
+        A.append(np.eye(nb) + (cond / np.linalg.norm(e, 2)) * (e + e.conj().T) / 2)
+    dA = ctx.to_dev(np.ascontiguousarray(np.stack(A).transpose(0, 2, 1)))
+    ctx.inverse_hpd_dev(dA, nb, 8, nb)
+    got = dA.download(np.complex128, (8, nb, nb)).transpose(0, 2, 1)
+    dA.free()
+    err = []
+    for a, x in zip(A, got):
+        al, r = a.astype(np.clongdouble), np.linalg.inv(a).astype(np.clongdouble)
+        for _ in range(3):
+            r = r @ (2 * np.eye(nb) - al @ r)
+        err.append([float(np.linalg.norm((y - r).astype(complex)) / np.linalg.norm(r.astype(complex)))
+                    for y in (x, _eliminate(a))])
+    e, ref = np.exp(np.mean(np.log(err), axis=0))
+    print(f"nb={nb} cond={cond:.0e}: {e:.2e}, pivot by pivot {ref:.2e}")
+    assert e < 2 * ref, (e, ref)
+
+
 class _Off:
     """A device buffer seen from a byte offset."""
 
