@@ -29,7 +29,9 @@ using chi0t::Problem;
 
 // The tiles of one call in launch order, and how the last of them are split
 // over the transitions: tiles t < full are whole; each of the rest is summed
-// in ks parts into `part`, which chi0_reduce_kernel adds in order.
+// in ks parts, which are added in order: by chi0_reduce_kernel from `part`, or,
+// where there is no room for them (part null), by one workgroup per tile that
+// runs the parts one after the other (chi0_parts_kernel).
 struct Split {
   int ntri;      // tiles per frequency
   long full;     // whole tiles
@@ -126,12 +128,46 @@ __global__ __launch_bounds__(chi0t::NT) void chi0_reduce_kernel(Problem P, Split
   chi0t::store_tile<CT, SPLIT>(P, bi, bj, w, acc);
 }
 
+// The split tiles without room for their parts: one workgroup per tile, the
+// parts in ascending order, the same sums as above.  Both accumulators take the
+// registers of one wave per SIMD.
+template <bool COLMAJOR, bool SPLIT, bool DMA>
+__global__ __launch_bounds__(chi0t::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
+chi0_parts_kernel(Problem P, Split S) {
+  __shared__ Lds<CT, CK, SPLIT> s;
+  const long t = S.full + blockIdx.x;
+  const int w = (int)(t / S.ntri);
+  int bi, bj;
+  chi0t::tri_index((int)(t % S.ntri), bi, bj);
+  const long nst = (P.n + CK - 1) / CK;
+  chi0t::Acc<CT / 32> acc, sum;
+#pragma unroll 1
+  for (int p = 0; p < S.ks; p++) {
+    chi0t::tile_sums<CT, CK, COLMAJOR, SPLIT, DMA>(P, bi, bj, w, nst * p / S.ks,
+                                                   nst * (p + 1) / S.ks, s, acc);
+    if (p == 0) {
+      sum = acc;
+      continue;
+    }
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        sum.re[a][b] += acc.re[a][b];
+        sum.im[a][b] += acc.im[a][b];
+      }
+  }
+  chi0t::store_tile<CT, SPLIT>(P, bi, bj, w, sum);
+}
+
 // How a call's tiles are split.  512 workgroups run at once (two per CU,
 // 65 KB of LDS each).  Whole rounds of 512 tiles run unsplit; the tiles of
 // the last, partial round are cut over the transitions so that they fill it:
 // 60 tiles (3,584 transitions, 256 columns, 6 frequencies) took 631 us whole
-// and take 144 us in 8 parts each, the reduction included.  A part keeps at least 8 K-slices, and 512 parts bound the workspace to
-// 32 MiB.  The rule depends on the sizes only, so the order of every sum does.
+// and take 144 us in 8 parts each, the reduction included.  A part keeps at
+// least 8 K-slices, and 512 parts bound the workspace to 32 MiB.  The rule
+// depends on the sizes only and both ways to run the parts add them in the same
+// order, so the order of every sum depends on the sizes only.
 constexpr int CSLOTS = 512;
 Split split_rule(long n, int nb, int nw) {
   const int nbt = (nb + CT - 1) / CT;
@@ -224,12 +260,20 @@ static void launch_one(hipStream_t st, const Problem &P, int colmajor) {
 }
 
 static void launch_tiles(hipStream_t st, const Problem &P, const Split &S, int colmajor, int split) {
-  const dim3 grid((unsigned)(S.full + (long)S.rem * S.ks)), block(chi0t::NT);
+  const dim3 grid((unsigned)(S.full + (S.part ? (long)S.rem * S.ks : 0))), block(chi0t::NT);
   auto go = [&](auto sp, auto dma) {
     constexpr bool SP = decltype(sp)::value, DMA = decltype(dma)::value;
-    if (colmajor) hipLaunchKernelGGL((chi0_kernel<true, SP, DMA>), grid, block, 0, st, P, S);
-    else hipLaunchKernelGGL((chi0_kernel<false, SP, DMA>), grid, block, 0, st, P, S);
-    if (S.rem) hipLaunchKernelGGL(chi0_reduce_kernel<SP>, dim3(S.rem), block, 0, st, P, S);
+    if (grid.x && colmajor)
+      hipLaunchKernelGGL((chi0_kernel<true, SP, DMA>), grid, block, 0, st, P, S);
+    else if (grid.x)
+      hipLaunchKernelGGL((chi0_kernel<false, SP, DMA>), grid, block, 0, st, P, S);
+    if (!S.rem) return;
+    if (S.part)
+      hipLaunchKernelGGL(chi0_reduce_kernel<SP>, dim3(S.rem), block, 0, st, P, S);
+    else if (colmajor)
+      hipLaunchKernelGGL((chi0_parts_kernel<true, SP, DMA>), dim3(S.rem), block, 0, st, P, S);
+    else
+      hipLaunchKernelGGL((chi0_parts_kernel<false, SP, DMA>), dim3(S.rem), block, 0, st, P, S);
   };
   if (split) go(std::true_type{}, std::false_type{});
   else if (chi0t::dma_ok(P.M)) go(std::false_type{}, std::true_type{});
@@ -447,7 +491,7 @@ int spx_col_scales(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void 
 int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                     const void *M, long ldm, int colmajor, int nw,
                     const void *wght, int precision, double alpha, double beta,
-                    void *chi, int ldchi, void *ws, int one) {
+                    void *chi, int ldchi, void *ws, size_t ws_bytes, int one) {
   SPX_CHECK(ctx, n >= 0 && nb > 0 && nw > 0, "chi0: bad sizes n=%ld nb=%d nw=%d", n, nb, nw);
   SPX_CHECK(ctx, ldchi >= nb, "chi0: ldchi=%d < nb=%d", ldchi, nb);
   SPX_CHECK(ctx, colmajor ? ldm >= n : ldm >= nb, "chi0: ldm=%ld too small", ldm);
@@ -467,19 +511,19 @@ int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
   const size_t sb = split ? scale_bytes(nb, nw, precision) : 0, pb = part_bytes(S);
   if (!ws && sb + pb) {
     SPX_CHECK(ctx, !sb || st == ctx->stream, "chi0: split form off the context stream needs a workspace");
-    // Tiles stay whole when the budget has no room for their parts, and off
-    // the context stream, whose buffer this is.
-    int rc = st == ctx->stream ? spx_chi0_buf(ctx, sb + pb, &ws) : SPEXHIP_E_NOMEM;
+    // the context's buffer, whose parts are left out when the budget has no
+    // room for them, and off the context stream
+    ws_bytes = st == ctx->stream ? sb + pb : 0;
+    int rc = ws_bytes ? spx_chi0_buf(ctx, ws_bytes, &ws) : SPEXHIP_OK;
     if (rc == SPEXHIP_E_NOMEM && pb) {
-      S.full += S.rem;
-      S.rem = 0;
-      S.ks = 1;
+      ws_bytes = sb;
       rc = sb ? spx_chi0_buf(ctx, sb, &ws) : SPEXHIP_OK;
     }
     if (rc) return rc;
   }
+  SPX_CHECK(ctx, ws_bytes >= sb, "chi0: workspace too small");
   double *scale = sb ? (double *)ws : nullptr;
-  S.part = (double2 *)((char *)ws + sb);
+  S.part = pb && ws_bytes >= sb + pb ? (double2 *)((char *)ws + sb) : nullptr;
   if (split) {
     int rc = spx_col_scales(ctx, st, n, nb, M, ldm, colmajor, nw, (const double *)wght, 1, scale);
     if (rc) return rc;
@@ -581,7 +625,8 @@ int spexhip_chi0_noalloc_dev(spexhip_ctx *ctx, long n, int nb, const void *M, lo
             "chi0_noalloc: chi is not a context allocation of the stated shape");
   SPX_HIP(ctx, hipSetDevice(ctx->device));
   return spx_chi0_launch(ctx, ctx->stream, n, nb, M, ldm, colmajor, nw, wght, precision,
-                         alpha, beta, chi, ldchi, ctx->noalloc_scales);
+                         alpha, beta, chi, ldchi, ctx->noalloc_scales,
+                         sizeof(double) * (SPEXHIP_NOALLOC_MAX_SCALES + 2 * CSLOTS * CT * CT));
 }
 
 int spexhip_pack_upper_d2h(spexhip_ctx *ctx, int nb, int nw, const void *X, int ldx,

@@ -96,14 +96,16 @@ int spx_noalloc_setup(spexhip_ctx *ctx);
 int spx_chi0_ozaki(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void *M, long ldm,
                    int colmajor, int nw, const void *wght, double alpha, double beta, void *chi,
                    int ldchi, size_t ws_limit);
-// ws: spx_chi0_ws_bytes bytes, 256-byte aligned (FP64 and split-FP32 forms);
-// nullptr takes the context's own buffer (the split-FP32 form then needs st
-// to be the context stream).  one: FP64 sums in one chain per output (see
-// chi0_one_kernel), without workspace.
+// ws: workspace, 256-byte aligned (FP64 and split-FP32 forms): column scales,
+// which it must hold, then the parts of split tiles, which run one after the
+// other if ws_bytes < spx_chi0_ws_bytes (the same sums).  nullptr takes the
+// context's own buffer (the split-FP32 form then needs st to be the context
+// stream).  one: FP64 sums in one chain per output (see chi0_one_kernel),
+// without workspace.
 int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                     const void *M, long ldm, int colmajor, int nw,
                     const void *wght, int precision, double alpha, double beta,
-                    void *chi, int ldchi, void *ws = nullptr, int one = 0);
+                    void *chi, int ldchi, void *ws = nullptr, size_t ws_bytes = 0, int one = 0);
 // Bytes of ws: column scales of the split-FP32 form and the parts of the
 // split tiles (non-decreasing in n, at most 32 MiB beside the scales).
 size_t spx_chi0_ws_bytes(long n, int nb, int nw, int precision);

@@ -112,7 +112,7 @@ int enqueue(spexhip_ctx *ctx, spexhip_qpipe *q) {
                                 d.nb, q->ws, q->wsb, q->flags + 1);
     else
       rc = spx_chi0_launch(ctx, st, np, d.nb, Mp, q->ldm, 0, d.nw, q->D, d.precision, d.alpha,
-                           beta, q->X, d.nb, q->ws);
+                           beta, q->X, d.nb, q->ws, q->wsb);
     if (rc) return rc;
   }
   rc = spx_dielectric(ctx, st, d.nb, d.nw, q->X, d.nb, d.vkind, d.vhalf_dev, q->E, d.nb, q->ws);

@@ -351,3 +351,39 @@ def test_ozaki_transitions_in_parts(ctx, n, nb, nw, beta):
         assert err.max() < 2 * 2 * 2.4e-10, (w, err.max())
     for b in (dM, dD, dX):
         b.free()
+
+
+@pytest.mark.parametrize("precision", [spexhip.PREC_FP64, spexhip.PREC_SPLIT_FP32])
+@pytest.mark.parametrize("n,nb,nw,col,off", [
+    (600, 130, 6, False, 0), (601, 130, 6, True, 0), (599, 129, 5, False, 8),
+    (600, 130, 100, False, 0),  # 512 whole tiles and 88 split ones
+    (5000, 70, 2, False, 0)])
+def test_split_tiles_same_sums_without_room_for_parts(precision, n, nb, nw, col, off):
+    """The parts of the split tiles in a context whose budget has no room for them (one workgroup
+    per tile runs them in turn) add up in the same order as the parts in memory: bit for bit the
+    result of a context without limit and of the call that allocates nothing."""
+    g = np.random.default_rng(n + nb + nw)
+    M = g.standard_normal((n, nb)) + 1j * g.standard_normal((n, nb))
+    D = g.standard_normal((nw, n))
+    X0 = g.standard_normal((nw, nb, nb)) + 1j * g.standard_normal((nw, nb, nb))
+    iu = np.triu_indices(nb)
+    out, budget = [], 0
+    for limit in (False, True):
+        with spexhip.Context(0, hbm_budget=budget) as c:
+            raw = c.alloc(M.nbytes + 16)
+            raw.upload(np.concatenate([np.zeros(off // 8), np.ascontiguousarray(M.T if col else M)
+                                       .view(np.float64).ravel()]))
+            dD, dX = c.to_dev(D), c.alloc(X0.nbytes)
+            room = c.mem_used()[0] + (1 << 20)
+            for call in (c.chi0_dev, c.chi0_noalloc_dev):
+                dX.upload(X0)
+                call(n, nb, _At(raw, off), n if col else nb, col, nw, dD, precision, dX, nb,
+                     alpha=1.7, beta=-0.3)
+                out.append(dX.download(np.complex128, (nw, nb, nb)).transpose(0, 2, 1)[:, iu[0], iu[1]])
+            if limit:
+                assert c.mem_used()[0] <= budget
+            else:
+                assert c.mem_used()[0] > room  # the parts
+                budget = room
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
