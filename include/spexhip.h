@@ -303,14 +303,15 @@ int spexhip_chi0_dev(spexhip_ctx *ctx, long n, int nb, const void *M_dev,
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): spexhip_chi0_dev with the same arguments and results,
  * bit for bit, but no hipMalloc, hipFree or other allocation.  The
- * split-FP32 column scales (nb*nw doubles, at most
- * SPEXHIP_NOALLOC_MAX_SCALES) and the partial sums of split tiles (32 MiB)
- * live in a fixed device array (33 MiB per GPU, held until the process
+ * split-FP32 column scales (nb*nw doubles) live in a fixed device array of
+ * SPEXHIP_NOALLOC_MAX_SCALES doubles (1 MiB per GPU, held until the process
  * ends) instead of a context buffer; nb*nw above that limit, and the Ozaki
- * form (its slice workspace is gigabytes), return SPEXHIP_E_INVALID.  All
- * calls on one GPU share that array: calls that overlap in time on one GPU
- * (other contexts or threads) race.  The array is rewritten by every call
- * before it is read.                                                       */
+ * form (its slice workspace is gigabytes), return SPEXHIP_E_INVALID.
+ * Split-FP32 calls on one GPU share that array: those that overlap in time on
+ * one GPU (other contexts or threads) race.  The array is rewritten by every
+ * call before it is read.  FP64 calls use no memory but their arguments.
+ * Where spexhip_chi0_dev sums parts of a tile in different workgroups (few
+ * tiles), this call runs them in one, which takes longer.                  */
 #define SPEXHIP_NOALLOC_MAX_SCALES 131072
 int spexhip_chi0_noalloc_dev(spexhip_ctx *ctx, long n, int nb, const void *M_dev,
                              long ldm, int colmajor, int nw, const void *wght_dev,

@@ -130,7 +130,8 @@ __global__ __launch_bounds__(chi0t::NT) void chi0_reduce_kernel(Problem P, Split
 
 // The split tiles without room for their parts: one workgroup per tile, the
 // parts in ascending order, the same sums as above.  Both accumulators take the
-// registers of one wave per SIMD.
+// registers of one wave per SIMD.  60 tiles of 3,584 transitions: 444 us (145 us
+// in 8 parts each, side by side); 196 tiles of 9,045: 1,103 us (995).
 template <bool COLMAJOR, bool SPLIT, bool DMA>
 __global__ __launch_bounds__(chi0t::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 chi0_parts_kernel(Problem P, Split S) {
@@ -429,14 +430,15 @@ size_t spx_chi0_ws_bytes(long n, int nb, int nw, int precision) {
   return scale_bytes(nb, nw, precision) + part_bytes(split_rule(n, nb, nw));
 }
 
-// Workspace of spexhip_chi0_noalloc_dev (column scales, then the parts of
-// split tiles): a fixed array in device memory (one copy per GPU, held until
-// the process ends) instead of a context allocation.  Host code never passes
-// `scratch` itself to a kernel (on the host its name is a stand-in, not a
-// device address); spx_noalloc_setup looks up the device address once per
-// context, with the context's device current, and the entry point passes
-// that address.
-static __device__ __align__(256) double scratch[SPEXHIP_NOALLOC_MAX_SCALES + 2 * CSLOTS * CT * CT];
+// Column scales of spexhip_chi0_noalloc_dev: a fixed array in device memory
+// (one copy per GPU, held until the process ends) instead of a context
+// allocation.  All contexts on a GPU share it, so nothing else goes there: the
+// FP64 form uses none of it and overlapping FP64 calls stay independent.  Host
+// code never passes `scratch` itself to a kernel (on the host its name is a
+// stand-in, not a device address); spx_noalloc_setup looks up the device
+// address once per context, with the context's device current, and the entry
+// point passes that address.
+static __device__ __align__(256) double scratch[SPEXHIP_NOALLOC_MAX_SCALES];
 
 int spx_noalloc_setup(spexhip_ctx *ctx) {
   void *ptr = nullptr;
@@ -491,7 +493,7 @@ int spx_col_scales(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void 
 int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                     const void *M, long ldm, int colmajor, int nw,
                     const void *wght, int precision, double alpha, double beta,
-                    void *chi, int ldchi, void *ws, size_t ws_bytes, int one) {
+                    void *chi, int ldchi, void *ws, size_t ws_bytes, int how) {
   SPX_CHECK(ctx, n >= 0 && nb > 0 && nw > 0, "chi0: bad sizes n=%ld nb=%d nw=%d", n, nb, nw);
   SPX_CHECK(ctx, ldchi >= nb, "chi0: ldchi=%d < nb=%d", ldchi, nb);
   SPX_CHECK(ctx, colmajor ? ldm >= n : ldm >= nb, "chi0: ldm=%ld too small", ldm);
@@ -503,13 +505,14 @@ int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                           ctx->ozaki_ws_limit);
   const int split = precision == SPEXHIP_PREC_SPLIT_FP32 && n > 0;
   Split S = split_rule(n, nb, nw);
-  if (one && !split) {
+  const bool one = (how & CHI0_ONE) && !split;
+  if (one) {
     S.full += S.rem;
     S.rem = 0;
     S.ks = 1;
   }
   const size_t sb = split ? scale_bytes(nb, nw, precision) : 0, pb = part_bytes(S);
-  if (!ws && sb + pb) {
+  if (!ws && sb + pb && !(how & CHI0_NO_PARTS)) {
     SPX_CHECK(ctx, !sb || st == ctx->stream, "chi0: split form off the context stream needs a workspace");
     // the context's buffer, whose parts are left out when the budget has no
     // room for them, and off the context stream
@@ -523,14 +526,15 @@ int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
   }
   SPX_CHECK(ctx, ws_bytes >= sb, "chi0: workspace too small");
   double *scale = sb ? (double *)ws : nullptr;
-  S.part = pb && ws_bytes >= sb + pb ? (double2 *)((char *)ws + sb) : nullptr;
+  const bool parts = pb && !(how & CHI0_NO_PARTS) && ws_bytes >= sb + pb;
+  S.part = parts ? (double2 *)((char *)ws + sb) : nullptr;
   if (split) {
     int rc = spx_col_scales(ctx, st, n, nb, M, ldm, colmajor, nw, (const double *)wght, 1, scale);
     if (rc) return rc;
   }
   Problem P{n, nb, nw, (const double2 *)M, ldm, (const double *)wght, (double2 *)chi,
             (long)ldchi, n == 0 ? 0.0 : alpha, beta, scale};
-  if (one && !split) launch_one(st, P, colmajor);
+  if (one) launch_one(st, P, colmajor);
   else launch_tiles(st, P, S, colmajor, split);
   SPX_LAUNCHED(ctx);
   return SPEXHIP_OK;
@@ -626,7 +630,7 @@ int spexhip_chi0_noalloc_dev(spexhip_ctx *ctx, long n, int nb, const void *M, lo
   SPX_HIP(ctx, hipSetDevice(ctx->device));
   return spx_chi0_launch(ctx, ctx->stream, n, nb, M, ldm, colmajor, nw, wght, precision,
                          alpha, beta, chi, ldchi, ctx->noalloc_scales,
-                         sizeof(double) * (SPEXHIP_NOALLOC_MAX_SCALES + 2 * CSLOTS * CT * CT));
+                         sizeof(double) * SPEXHIP_NOALLOC_MAX_SCALES, CHI0_NO_PARTS);
 }
 
 int spexhip_pack_upper_d2h(spexhip_ctx *ctx, int nb, int nw, const void *X, int ldx,

@@ -37,7 +37,8 @@ struct spexhip_ctx {
   // and batches carry their own)
   void *chi0_ws = nullptr;
   size_t chi0_ws_bytes = 0;
-  // device address of the fixed workspace of spexhip_chi0_noalloc_dev on this context's device (set at creation)
+  // device address of the fixed column-scale array of
+  // spexhip_chi0_noalloc_dev on this context's device (set at creation)
   void *noalloc_scales = nullptr;
   // largest slice workspace of the Ozaki form (frequencies are grouped to fit)
   size_t ozaki_ws_limit = (size_t)24 << 30;
@@ -88,7 +89,7 @@ int spx_scratch(spexhip_ctx *ctx, size_t bytes, void **p);
 int spx_chi0_buf(spexhip_ctx *ctx, size_t bytes, void **p);
 // Is `p` (or p+bytes-1) inside an allocation of this context?
 bool spx_owns(spexhip_ctx *ctx, const void *p, size_t bytes);
-// Looks up the device address of the no-alloc workspace (chi0.hip)
+// Looks up the device address of the no-alloc column-scale array (chi0.hip)
 // on the current device and stores it in ctx->noalloc_scales.
 int spx_noalloc_setup(spexhip_ctx *ctx);
 
@@ -100,12 +101,14 @@ int spx_chi0_ozaki(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void 
 // which it must hold, then the parts of split tiles, which run one after the
 // other if ws_bytes < spx_chi0_ws_bytes (the same sums).  nullptr takes the
 // context's own buffer (the split-FP32 form then needs st to be the context
-// stream).  one: FP64 sums in one chain per output (see chi0_one_kernel),
-// without workspace.
+// stream).  how: CHI0_ONE, FP64 sums in one chain per output (see
+// chi0_one_kernel), without workspace; CHI0_NO_PARTS, the parts one after the
+// other whatever the workspace.
+enum { CHI0_ONE = 1, CHI0_NO_PARTS = 2 };
 int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                     const void *M, long ldm, int colmajor, int nw,
                     const void *wght, int precision, double alpha, double beta,
-                    void *chi, int ldchi, void *ws = nullptr, size_t ws_bytes = 0, int one = 0);
+                    void *chi, int ldchi, void *ws = nullptr, size_t ws_bytes = 0, int how = 0);
 // Bytes of ws: column scales of the split-FP32 form and the parts of the
 // split tiles (non-decreasing in n, at most 32 MiB beside the scales).
 size_t spx_chi0_ws_bytes(long n, int nb, int nw, int precision);

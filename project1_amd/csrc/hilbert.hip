@@ -139,10 +139,10 @@ int spexhip_chi0_cplx_dev(spexhip_ctx *ctx, long n, int nb, const void *M, long 
   int rc = spx_scratch(ctx, cbytes, &T);
   if (rc) return rc;
   rc = spx_chi0_launch(ctx, ctx->stream, n, nb, M, ldm, colmajor, nw, Dr, precision, alpha, 0.0,
-                       chi, ldchi, nullptr, 0, 1);
+                       chi, ldchi, nullptr, 0, CHI0_ONE);
   if (!rc)
     rc = spx_chi0_launch(ctx, ctx->stream, n, nb, M, ldm, colmajor, nw, Di, precision, alpha, 0.0,
-                         T, ldchi, nullptr, 0, 1);
+                         T, ldchi, nullptr, 0, CHI0_ONE);
   if (rc) return rc;
   const long npack = (long)nb * (nb + 1) / 2;
   hipLaunchKernelGGL(cplx_combine_kernel, dim3((unsigned)((npack + 255) / 256), nw), dim3(256), 0,

@@ -70,3 +70,26 @@ def test_noalloc_refusals():
         assert e.value.code == spexhip.E_INVALID and "exceeds" in str(e.value)
         for d in (dM, dW, chi):
             d.free()
+
+
+def test_noalloc_fp64_calls_of_two_contexts_overlap():
+    """FP64 calls use no memory but their arguments: calls of two contexts whose kernels run at
+    the same time, on sizes whose tiles are split, give each its own result."""
+    with spexhip.Context(0) as a, spexhip.Context(0) as b:
+        jobs = []
+        for ctx, seed in ((a, 21), (b, 22)):
+            c, dM, dW = _case(ctx, 6, 8, 40, 200, 6, seed)
+            n, nb, nw = c.M.shape[0], 200, 6
+            want, got = (ctx.alloc(16 * nb * nb * nw).zero() for _ in range(2))
+            ctx.chi0_dev(n, nb, dM, nb, False, nw, dW, spexhip.PREC_FP64, want, nb, alpha=2.0)
+            ctx.sync()
+            jobs.append((ctx, n, nb, nw, dM, dW, want, got))
+        for _ in range(20):
+            for ctx, n, nb, nw, dM, dW, want, got in jobs:  # asynchronous, two streams
+                ctx.chi0_noalloc_dev(n, nb, dM, nb, False, nw, dW, spexhip.PREC_FP64, got, nb,
+                                     alpha=2.0)
+            for ctx, n, nb, nw, dM, dW, want, got in jobs:
+                iu = np.triu_indices(nb)
+                x, y = (v.download(np.complex128, (nw, nb, nb))[:, iu[1], iu[0]]
+                        for v in (want, got))
+                np.testing.assert_array_equal(y, x)
