@@ -512,11 +512,13 @@ int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
     S.ks = 1;
   }
   const size_t sb = split ? scale_bytes(nb, nw, precision) : 0, pb = part_bytes(S);
+  std::unique_lock<std::mutex> own;  // of the context's buffer, until the launches are enqueued
   if (!ws && sb + pb && !(how & CHI0_NO_PARTS)) {
     SPX_CHECK(ctx, !sb || st == ctx->stream, "chi0: split form off the context stream needs a workspace");
     // the context's buffer, whose parts are left out when the budget has no
     // room for them, and off the context stream
     ws_bytes = st == ctx->stream ? sb + pb : 0;
+    if (ws_bytes) own = std::unique_lock<std::mutex>(ctx->chi0_mu);
     int rc = ws_bytes ? spx_chi0_buf(ctx, ws_bytes, &ws) : SPEXHIP_OK;
     if (rc == SPEXHIP_E_NOMEM && pb) {
       ws_bytes = sb;

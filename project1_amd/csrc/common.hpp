@@ -34,7 +34,10 @@ struct spexhip_ctx {
   size_t scratch_bytes = 0;
   // workspace of the FP64 and split-FP32 chi0 forms (column scales, parts of
   // split tiles) for calls on the context stream (grown on demand; pipelines
-  // and batches carry their own)
+  // and batches carry their own); chi0_mu is held from its lookup until the
+  // launches that use it are enqueued, so that another thread's call neither
+  // frees it in between nor puts its kernels between theirs
+  std::mutex chi0_mu;
   void *chi0_ws = nullptr;
   size_t chi0_ws_bytes = 0;
   // device address of the fixed column-scale array of
@@ -85,7 +88,7 @@ int spx_aux_stream(spexhip_ctx *ctx);
 int spx_free(spexhip_ctx *ctx, void *p);
 // Context-owned scratch of at least `bytes` (contents undefined).
 int spx_scratch(spexhip_ctx *ctx, size_t bytes, void **p);
-// Context-owned workspace of the chi0 forms (context stream only).
+// Context-owned workspace of the chi0 forms (context stream only; chi0_mu held).
 int spx_chi0_buf(spexhip_ctx *ctx, size_t bytes, void **p);
 // Is `p` (or p+bytes-1) inside an allocation of this context?
 bool spx_owns(spexhip_ctx *ctx, const void *p, size_t bytes);

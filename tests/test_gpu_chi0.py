@@ -387,3 +387,46 @@ def test_split_tiles_same_sums_without_room_for_parts(precision, n, nb, nw, col,
                 budget = room
     for o in out[1:]:
         np.testing.assert_array_equal(o, out[0])
+
+
+def test_pair_sums_of_two_threads_on_one_context():
+    """Two host threads call chi0_dev on one context, with workspaces of growing and of differing
+    size: every result equals, bit for bit, the one of a call made alone."""
+    import threading
+
+    sizes = [(200, 70, 1), (600, 130, 6), (1500, 90, 3), (3000, 250, 6)]
+    with spexhip.Context(0) as ref, spexhip.Context(0) as c:
+        jobs = []
+        for i, (n, nb, nw) in enumerate(sizes):
+            g = np.random.default_rng(i)
+            M = g.standard_normal((n, nb)) + 1j * g.standard_normal((n, nb))
+            D = -g.uniform(0.1, 2.0, (nw, n))
+            iu = np.triu_indices(nb)
+            for prec in (spexhip.PREC_FP64, spexhip.PREC_SPLIT_FP32):
+                dM, dD, dX = ref.to_dev(M), ref.to_dev(D), ref.alloc(16 * nb * nb * nw)
+                ref.chi0_dev(n, nb, dM, nb, False, nw, dD, prec, dX, nb)
+                want = dX.download(np.complex128, (nw, nb, nb))[:, iu[1], iu[0]]
+                jobs.append((n, nb, nw, prec, c.to_dev(M), c.to_dev(D), iu, want))
+        bad = []
+
+        def work(order):
+            try:
+                outs = [c.alloc(16 * j[1] * j[1] * j[2]) for j in jobs]
+                for _ in range(8):
+                    for k in order:
+                        n, nb, nw, prec, dM, dD = jobs[k][:6]
+                        c.chi0_dev(n, nb, dM, nb, False, nw, dD, prec, outs[k], nb)
+                for k, (n, nb, nw, prec, _, _, iu, want) in enumerate(jobs):
+                    got = outs[k].download(np.complex128, (nw, nb, nb))[:, iu[1], iu[0]]
+                    if not np.array_equal(got, want):
+                        bad.append((n, nb, nw, prec))
+            except Exception as e:  # reported by the main thread
+                bad.append(e)
+
+        order = list(range(len(jobs)))
+        ts = [threading.Thread(target=work, args=(o,)) for o in (order, order[::-1])]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert not bad, bad
