@@ -40,7 +40,7 @@ static void trim_cache(spexhip_ctx *ctx) {
   for (auto &kv : blocks) (void)hipFree(kv.second);
 }
 
-int spx_alloc(spexhip_ctx *ctx, size_t bytes, void **p) {
+static int alloc_once(spexhip_ctx *ctx, size_t bytes, void **p) {
   const size_t cls = size_class(bytes);
   {
     std::lock_guard<std::mutex> g(ctx->mu);
@@ -76,6 +76,23 @@ int spx_alloc(spexhip_ctx *ctx, size_t bytes, void **p) {
   std::lock_guard<std::mutex> g(ctx->mu);
   ctx->allocs[*p] = {bytes, cls};
   return SPEXHIP_OK;
+}
+
+// Gives the pair sum's workspace back; false if there is none.
+static bool release_chi0_ws(spexhip_ctx *ctx) {
+  std::lock_guard<std::mutex> g(ctx->chi0_mu);
+  if (!ctx->chi0_ws || hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  spx_free(ctx, ctx->chi0_ws);
+  ctx->chi0_ws = nullptr;
+  ctx->chi0_ws_bytes = 0;
+  return true;
+}
+
+// The pair sum keeps up to 32 MiB of parts between calls, which it can do
+// without: what does not fit beside them takes their place.
+int spx_alloc(spexhip_ctx *ctx, size_t bytes, void **p) {
+  const int rc = alloc_once(ctx, bytes, p);
+  return rc == SPEXHIP_E_NOMEM && release_chi0_ws(ctx) ? alloc_once(ctx, bytes, p) : rc;
 }
 
 // The caller guarantees that no queued work still uses the block.
@@ -143,7 +160,7 @@ int spx_chi0_buf(spexhip_ctx *ctx, size_t bytes, void **p) {
     ctx->chi0_ws_bytes = 0;
     if (rc) return rc;
   }
-  int rc = spx_alloc(ctx, bytes, &ctx->chi0_ws);
+  int rc = alloc_once(ctx, bytes, &ctx->chi0_ws);
   if (rc) return rc;
   ctx->chi0_ws_bytes = bytes;
   *p = ctx->chi0_ws;

@@ -430,3 +430,25 @@ def test_pair_sums_of_two_threads_on_one_context():
         for t in ts:
             t.join()
         assert not bad, bad
+
+
+@pytest.mark.parametrize("precision", [spexhip.PREC_FP64, spexhip.PREC_SPLIT_FP32])
+def test_parts_give_way_to_allocations(precision):
+    """The parts that a pair sum leaves in the context count against its budget, but an allocation
+    that fits without them succeeds, and the next pair sum gives the same bits."""
+    n, nb, nw = 600, 130, 6  # 9 MiB of parts
+    g = np.random.default_rng(5)
+    M = g.standard_normal((n, nb)) + 1j * g.standard_normal((n, nb))
+    D = g.standard_normal((nw, n))
+    iu = np.triu_indices(nb)
+    with spexhip.Context(0, hbm_budget=24 << 20) as c:
+        dM, dD, dX = c.to_dev(M), c.to_dev(D), c.alloc(16 * nb * nb * nw)
+        free = (24 << 20) - c.mem_used()[0]
+        out = []
+        for _ in range(2):
+            c.chi0_dev(n, nb, dM, nb, False, nw, dD, precision, dX, nb)
+            out.append(dX.download(np.complex128, (nw, nb, nb))[:, iu[1], iu[0]])
+            if len(out) == 1:
+                big = c.alloc(free * 7 // 8)  # rounded up to a size class
+        np.testing.assert_array_equal(out[1], out[0])
+        big.free()
