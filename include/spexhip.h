@@ -68,7 +68,8 @@ int spexhip_sync(spexhip_ctx *ctx);
 int spexhip_mem_used(spexhip_ctx *ctx, size_t *used, size_t *budget);
 
 /* Largest slice workspace the Ozaki chi0 form may use (default 24 GiB); the
- * frequencies are processed in groups that fit.                            */
+ * frequencies are processed in groups that fit.  The order of that form's
+ * FP64 sums, and so their last bits, depends on the room.                  */
 int spexhip_set_workspace_limit(spexhip_ctx *ctx, size_t bytes);
 /* Event-timed phases of the last Ozaki chi0 call: prep = weights, scales
  * and slices of the first frequency group; rank = rank-k kernels (and the
@@ -817,7 +818,11 @@ typedef struct {
   int kpacket;
 } spexhip_qdesc;
 
-/* HBM bytes a pipeline of this shape allocates (admission by footprint). */
+/* HBM bytes a pipeline of this shape needs (admission by footprint).  Where
+ * the budget has room, creation takes up to 32 MiB more for the FP64 and
+ * split-FP32 forms, which then sum parts of a tile in different workgroups
+ * (the same results, sooner); the int8 form's parts (16 MiB at most) are in
+ * the footprint, and left out where only that makes it fit.                */
 int spexhip_qpipe_footprint(const spexhip_qdesc *desc, size_t *bytes);
 int spexhip_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, spexhip_qpipe **qp);
 /* Enqueue one run (asynchronous).  use_graph: capture on the first call,

@@ -300,19 +300,28 @@ int spexhip_batch_create(spexhip_ctx *ctx, int nq, const spexhip_qdesc *descs, i
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     if (e != hipSuccess) rc = spx_seterr(ctx, SPEXHIP_E_DEVICE, "batch: stream/event creation failed");
   }
-  // Ozaki: one slice workspace per stream, sized for its largest packet
-  for (int s = 0; s < b->nstream && !rc && ozaki; s++) {
-    size_t need = 0;
-    for (const auto &q : b->q)
-      if (q.s == s) {
-        const long n = (long)std::min(kpacket, q.d.nk) * q.d.nocc * q.d.nunocc;
-        need = std::max(need, spx_ozaki_ws_bytes(n, q.d.nb, q.d.nw,
-                                                 q.d.ozaki_group > 0 ? std::min(q.d.ozaki_group, q.d.nw) : q.d.nw));
-      }
-    void *raw = nullptr;
-    grab(need + 1024, &raw);  // the slice kernels want a 1 KB aligned workspace
-    b->ozws[s] = (void *)(((uintptr_t)raw + 1023) & ~(uintptr_t)1023);
-    b->ozwsb[s] = need;
+  // Ozaki: one slice workspace per stream, sized for its largest packet, with
+  // room for the parts of split tiles unless the budget has none
+  const size_t nowned = b->owned.size();
+  for (bool parts : {true, false}) {
+    if (rc || !ozaki) break;
+    for (int s = 0; s < b->nstream && !rc; s++) {
+      size_t need = 0;
+      for (const auto &q : b->q)
+        if (q.s == s) {
+          const long n = (long)std::min(kpacket, q.d.nk) * q.d.nocc * q.d.nunocc;
+          need = std::max(need, spx_ozaki_ws_bytes(n, q.d.nb, q.d.nw,
+                                                   q.d.ozaki_group > 0 ? std::min(q.d.ozaki_group, q.d.nw) : q.d.nw,
+                                                   parts));
+        }
+      void *raw = nullptr;
+      grab(need + 1024, &raw);  // the slice kernels want a 1 KB aligned workspace
+      b->ozws[s] = (void *)(((uintptr_t)raw + 1023) & ~(uintptr_t)1023);
+      b->ozwsb[s] = need;
+    }
+    if (rc != SPEXHIP_E_NOMEM || !parts) break;
+    for (; b->owned.size() > nowned; b->owned.pop_back()) spx_free(ctx, b->owned.back());
+    rc = SPEXHIP_OK;
   }
   // tile configuration (grouped kernel): given, or timed on packet 0 with
   // every q's K scaled down by one common factor (so the longest-first

@@ -551,9 +551,9 @@ static size_t ozk_part_bytes(long n, int nb, int nwg) {
 }
 
 // Workspace of the Ozaki form when nwg frequencies are sliced at a time.
-size_t spx_ozaki_ws_bytes(long n, int nb, int nw, int nwg) {
+size_t spx_ozaki_ws_bytes(long n, int nb, int nw, int nwg, bool parts) {
   return ozaki_fixed_bytes(n, nb, nw) + spx_ozaki_slice_bytes(n, nb) * (size_t)nwg +
-         ozk_part_bytes(n, nb, nwg);
+         (parts ? ozk_part_bytes(n, nb, nwg) : 0);
 }
 
 // Asynchronous Ozaki chi0 on stream st with caller workspace ws (ws_bytes >=
@@ -688,10 +688,11 @@ int spx_chi0_ozaki(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void 
   const size_t fixed = ozaki_fixed_bytes(n, nb, nw) + 1024, sb = spx_ozaki_slice_bytes(n, nb);
   int nwg = nw;
   while (nwg > 1 && fixed + sb * (size_t)nwg > ws_limit) nwg--;
-  size_t wsb = fixed + sb * (size_t)nwg;
-  if (wsb + ozk_part_bytes(n, nb, nwg) <= ws_limit) wsb += ozk_part_bytes(n, nb, nwg);
+  const size_t lean = fixed + sb * (size_t)nwg, pb = ozk_part_bytes(n, nb, nwg);
+  size_t wsb = lean + pb <= ws_limit ? lean + pb : lean;
   void *ws;
   int rc = spx_scratch(ctx, wsb, &ws);
+  if (rc == SPEXHIP_E_NOMEM && wsb > lean) rc = spx_scratch(ctx, wsb = lean, &ws);
   if (rc) return rc;
   int *err = (int *)((char *)ws + wsb - 1024);
   SPX_HIP(ctx, hipMemsetAsync(err, 0, sizeof(int), st));

@@ -114,6 +114,6 @@ int spx_chi0_launch(spexhip_ctx *ctx, hipStream_t st, long n, int nb,
                     void *chi, int ldchi, void *ws = nullptr, size_t ws_bytes = 0, int how = 0);
 // Bytes of ws: column scales of the split-FP32 form and the parts of the
 // split tiles (non-decreasing in n, at most 32 MiB beside the scales).
-size_t spx_chi0_ws_bytes(long n, int nb, int nw, int precision);
+size_t spx_chi0_ws_bytes(long n, int nb, int nw, int precision);  // with the parts
 // Bytes of the column scales of one problem.
 size_t spx_split_ws_bytes(int nb, int nw);

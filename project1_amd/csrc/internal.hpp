@@ -11,7 +11,8 @@ int spx_weights_launch(spexhip_ctx *ctx, hipStream_t st, int nk, int nocc, int n
 // grouped chi0 (persistent, many problems)
 int spx_group_launch(spexhip_ctx *ctx, hipStream_t st, const spexhip_group *g);
 // chi0 Ozaki form
-size_t spx_ozaki_ws_bytes(long n, int nb, int nw, int nwg);
+// parts: with room for the parts of tiles whose chunks are split
+size_t spx_ozaki_ws_bytes(long n, int nb, int nw, int nwg, bool parts = true);
 int spx_chi0_ozaki_async(spexhip_ctx *ctx, hipStream_t st, long n, int nb, const void *M,
                          long ldm, int colmajor, int nw, const void *wght, double alpha,
                          double beta, void *chi, int ldchi, void *ws, size_t ws_bytes,
@@ -38,6 +39,11 @@ int spx_inverse(spexhip_ctx *ctx, hipStream_t st, int nb, int nw, void *X, long 
                 int *flag, double *logdet_parts, int general = 0);
 int spx_screen(spexhip_ctx *ctx, hipStream_t st, int nb, int nw, const void *Einv, long lde,
                int vkind, const void *vh, void *W, long ldw, void *tmp);
+// a q pipeline: its device bytes with or without room for the parts of the pair
+// sum's split tiles, and its creation; with parts, they are left out where the
+// context has no room for them
+size_t spx_qpipe_bytes(const spexhip_qdesc &d, bool parts);
+int spx_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, bool parts, spexhip_qpipe **out);
 // packing and fills
 int spx_pack_upper(spexhip_ctx *ctx, hipStream_t st, int nb, int nw, const void *X, long ldx,
                    void *P);

@@ -43,8 +43,9 @@ int packet_k(const spexhip_qdesc &d) {
   return d.kpacket > 0 && d.kpacket < d.nk ? d.kpacket : (d.nk > 0 ? d.nk : 1);
 }
 
-// Buffers are sized for one packet of packet_k(d) k-points.
-Sizes sizes_of(const spexhip_qdesc &d) {
+// Buffers are sized for one packet of packet_k(d) k-points.  parts: with room
+// for the parts of the pair sum's split tiles.
+Sizes sizes_of(const spexhip_qdesc &d, bool parts) {
   Sizes s{};
   const int kp = packet_k(d);
   const long n = (long)kp * d.nocc * d.nunocc;
@@ -55,9 +56,10 @@ Sizes sizes_of(const spexhip_qdesc &d) {
   ws = std::max(ws, spx_inverse_ws(d.nb, d.nw));
   ws = std::max(ws, 16 * (size_t)d.nb * (d.nb + 1) / 2 * d.nw);  // packing
   if (d.precision != SPEXHIP_PREC_OZAKI_INT8)
-    ws = std::max(ws, spx_chi0_ws_bytes(n, d.nb, d.nw, d.precision));
+    ws = std::max(ws, parts ? spx_chi0_ws_bytes(n, d.nb, d.nw, d.precision)
+                            : spx_split_ws_bytes(d.nb, d.nw));
   if (d.precision == SPEXHIP_PREC_OZAKI_INT8)
-    ws = std::max(ws, spx_ozaki_ws_bytes(n, d.nb, d.nw, std::min(d.nw, d.ozaki_group > 0 ? d.ozaki_group : d.nw)));
+    ws = std::max(ws, spx_ozaki_ws_bytes(n, d.nb, d.nw, std::min(d.nw, d.ozaki_group > 0 ? d.ozaki_group : d.nw), parts));
   if (d.mt_plan) ws = std::max(ws, spx_wfprod_mt_ws(d.mt_plan, kp, d.nocc, d.nunocc));
   if (d.pw_plan) ws = std::max(ws, spx_wfprod_pw_ws_core(d.pw_plan, d.nocc, d.nunocc));
   s.ws = align256(ws);
@@ -133,15 +135,11 @@ void destroy(spexhip_ctx *ctx, spexhip_qpipe *q) {
 
 }  // namespace
 
-extern "C" {
-
-int spexhip_qpipe_footprint(const spexhip_qdesc *d, size_t *bytes) {
-  if (!d || !bytes) return SPEXHIP_E_INVALID;
-  *bytes = footprint_of(sizes_of(*d));
-  return SPEXHIP_OK;
+size_t spx_qpipe_bytes(const spexhip_qdesc &d, bool parts) {
+  return footprint_of(sizes_of(d, parts));
 }
 
-int spexhip_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, spexhip_qpipe **out) {
+int spx_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, bool parts, spexhip_qpipe **out) {
   if (!ctx || !desc || !out) return SPEXHIP_E_INVALID;
   *out = nullptr;
   const spexhip_qdesc &d = *desc;
@@ -171,29 +169,34 @@ int spexhip_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, spexhip_qp
     q->k2.assign(d.k2, d.k2 + d.nk);
     if (d.pw_plan) q->g2.assign(d.g2, d.g2 + 3 * d.nk);
   }
-  const Sizes s = sizes_of(d);
-  q->footprint = footprint_of(s);
-  int rc = SPEXHIP_OK;
-  auto grab = [&](size_t bytes, void **p) {
-    if (rc) return;
-    rc = spx_alloc(ctx, bytes, p);
-    if (!rc) q->owned.push_back(*p);
-  };
-  if (d.M_dev) {
-    q->M = const_cast<void *>(d.M_dev);
-    q->ldm = d.ldm;
-  } else {
-    grab(s.M, &q->M);
-    q->ownM = true;
-    q->ldm = d.nb;
-  }
-  grab(s.D, &q->D);
-  grab(s.X, &q->X);
-  grab(s.X, &q->E);
-  grab(s.ws, &q->ws);
-  q->wsb = s.ws;
+  q->ldm = d.M_dev ? d.ldm : d.nb;
+  q->ownM = !d.M_dev;
   void *tab = nullptr;
-  grab(s.tab, &tab);
+  auto reserve = [&](const Sizes &s) {
+    int rc = SPEXHIP_OK;
+    auto grab = [&](size_t bytes, void **p) {
+      if (rc) return;
+      rc = spx_alloc(ctx, bytes, p);
+      if (!rc) q->owned.push_back(*p);
+    };
+    if (d.M_dev) q->M = const_cast<void *>(d.M_dev);
+    else grab(s.M, &q->M);
+    grab(s.D, &q->D);
+    grab(s.X, &q->X);
+    grab(s.X, &q->E);
+    grab(s.ws, &q->ws);
+    grab(s.tab, &tab);
+    q->wsb = s.ws;
+    q->footprint = footprint_of(s);
+    return rc;
+  };
+  const Sizes lean = sizes_of(d, false), full = parts ? sizes_of(d, true) : lean;
+  int rc = reserve(full);
+  if (rc == SPEXHIP_E_NOMEM && full.ws > lean.ws) {  // without room for the parts
+    for (void *p : q->owned) spx_free(ctx, p);
+    q->owned.clear();
+    rc = reserve(lean);
+  }
   if (rc) {
     destroy(ctx, q);
     return rc;
@@ -229,6 +232,20 @@ int spexhip_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, spexhip_qp
   }
   *out = q;
   return SPEXHIP_OK;
+}
+
+extern "C" {
+
+// FP64 and split-FP32 sums are the same with and without the parts, so they
+// count as optional there; the int8 form adds up in another order.
+int spexhip_qpipe_footprint(const spexhip_qdesc *d, size_t *bytes) {
+  if (!d || !bytes) return SPEXHIP_E_INVALID;
+  *bytes = spx_qpipe_bytes(*d, d->precision == SPEXHIP_PREC_OZAKI_INT8);
+  return SPEXHIP_OK;
+}
+
+int spexhip_qpipe_create(spexhip_ctx *ctx, const spexhip_qdesc *desc, spexhip_qpipe **out) {
+  return spx_qpipe_create(ctx, desc, true, out);
 }
 
 int spexhip_qpipe_launch(spexhip_ctx *ctx, spexhip_qpipe *q, int use_graph) {

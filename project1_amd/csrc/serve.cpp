@@ -37,7 +37,8 @@ struct Req {
   long id = 0;
   spexhip_qdesc d{};
   std::vector<int> k1, k2, g2;
-  size_t footprint = 0;
+  size_t footprint = 0;  // device bytes reserved for it
+  size_t lean = 0, full = 0;  // without, with the parts of the pair sum's split tiles
   int state = 0;  // 0 queued, 1 running, 2 done, 3 failed
   int status = SPEXHIP_OK;
   std::string err;
@@ -106,10 +107,12 @@ static void scheduler(spexhip_server *s) {
       }
       const long id = *it;
       it = s->queue.erase(it);
+      if (r->d.precision != SPEXHIP_PREC_OZAKI_INT8 && s->used + r->full <= s->budget)
+        r->footprint = r->full;
       s->used += r->footprint;
       s->peak_used = std::max(s->peak_used, s->used);
       lk.unlock();  // pipeline creation allocates and uploads; other clients may submit
-      int rc = spexhip_qpipe_create(s->ctx, &r->d, &r->qp);
+      int rc = spx_qpipe_create(s->ctx, &r->d, r->footprint == r->full, &r->qp);
       if (!rc) rc = spexhip_qpipe_launch(s->ctx, r->qp, 0);
       lk.lock();
       r->t_start = Clock::now();
@@ -170,7 +173,12 @@ int spexhip_server_submit(spexhip_server *s, const spexhip_qdesc *d, long *id) {
     r->d.k2 = r->k2.empty() ? nullptr : r->k2.data();
     r->d.g2 = r->g2.empty() ? nullptr : r->g2.data();
   }
-  spexhip_qpipe_footprint(&r->d, &r->footprint);
+  // the int8 sums depend on whether the parts have room, so that is settled by
+  // the server's budget alone; the other forms take it at admission
+  const bool ozaki = r->d.precision == SPEXHIP_PREC_OZAKI_INT8;
+  r->lean = spx_qpipe_bytes(r->d, false);
+  r->full = spx_qpipe_bytes(r->d, true);
+  r->footprint = ozaki && r->full <= s->budget ? r->full : r->lean;
   if (r->footprint > s->budget)
     return spx_seterr(s->ctx, SPEXHIP_E_NOMEM,
                       "server: request footprint %zu exceeds the server budget %zu", r->footprint,

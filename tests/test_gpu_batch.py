@@ -109,3 +109,26 @@ def test_batch_ozaki_matches_per_q_and_footprint(lattice):
     b.destroy()
     for r in reqs:
         r.free()
+
+
+def test_batch_ozaki_budget_without_room_for_parts():
+    """int8 form on two q-points whose few tiles are split: a budget that holds the batch but not
+    the parts gives the same pair sums within 1e-8 (another order of the FP64 sums)."""
+    out, budget = [], 0
+    for _ in range(2):
+        with spexhip.Context(0, hbm_budget=budget) as c:
+            lat = serving.Lattice(c, nocc=4, nunocc=12, lcut=2, nrad=2, gcut=3.1,
+                                  nfft=(16, 16, 16), max_atoms=3, nb_max=100, ipw_target=40, seed=8)
+            reqs = [serving.Request(lat, serving.Spec(nmesh=3, nb=100, nw=3, seed=70 + i, iq=1 + i),
+                                    spexhip.PREC_OZAKI_INT8) for i in range(2)]
+            b = spexhip.Batch(c, [r.desc for r in reqs], kpacket=27)
+            used = c.mem_used()[0]
+            b.launch()
+            b.wait()
+            out.append([b.result(i, einv=False)[0] for i in range(2)])
+            b.destroy()
+        print(f"batch: {used} of {budget}")
+        assert not budget or used <= budget
+        budget = used - (1 << 20)
+    for x, y in zip(*out):
+        assert max(normwise(x, y)) < 1e-8

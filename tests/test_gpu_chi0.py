@@ -452,3 +452,37 @@ def test_parts_give_way_to_allocations(precision):
                 big = c.alloc(free * 7 // 8)  # rounded up to a size class
         np.testing.assert_array_equal(out[1], out[0])
         big.free()
+
+
+@pytest.mark.parametrize("n,nb,nw,group", [(4096, 130, 3, 3), (2000, 250, 6, 6), (17000, 64, 4, 1)])
+def test_ozaki_without_room_for_parts(n, nb, nw, group):
+    """int8 form where the parts of its split tiles do not fit: a workspace limit that holds
+    `group` frequencies' slices but not their parts, and a context budget that does not hold the
+    parts.  Whole tiles then, the same sums in another order: each real sum of two products per
+    transition of factors represented to 2.4e-10 s(I) s(J)."""
+    g = np.random.default_rng(n + nb)
+    M = g.standard_normal((n, nb)) + 1j * g.standard_normal((n, nb))
+    D = -g.uniform(0.1, 2.0, (nw, n))
+    iu = np.triu_indices(nb)
+    slices = 8 * (-(-n // 64) * 64) * (-(-nb // 64) * 64)  # one frequency's
+
+    def run(budget=0, limit=None):
+        with spexhip.Context(0, hbm_budget=budget) as c:
+            if limit:
+                c.set_workspace_limit(limit)
+            dM, dD, dX = c.to_dev(M), c.to_dev(D), c.alloc(16 * nb * nb * nw)
+            c.chi0_dev(n, nb, dM, nb, False, nw, dD, spexhip.PREC_OZAKI_INT8, dX, nb)
+            got = dX.download(np.complex128, (nw, nb, nb)).transpose(0, 2, 1)
+            for w in range(nw):
+                ref = (M * D[w][:, None]).T @ M.conj()
+                B = np.sqrt(np.abs(D[w]))[:, None] * M
+                sc = np.maximum(np.abs(B.real), np.abs(B.imag)).max(axis=0)
+                err = np.abs(got[w] - ref)[iu] / (n * np.outer(sc, sc)[iu])
+                assert err.max() < 2 * 2 * 2.4e-10, (w, err.max())
+            return c.mem_used()[0], c.chi0_phase_ms()[2]
+
+    full, _ = run()
+    lean, groups = run(limit=group * slices + (1 << 20))
+    assert lean < full and groups == -(-nw // group)
+    if group == nw:  # all frequencies at once fit the budget
+        assert run(budget=lean + (1 << 18))[0] <= lean + (1 << 18)
