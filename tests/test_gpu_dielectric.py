@@ -277,8 +277,8 @@ def test_inverse_at_panel_edges(ctx, nb, ld):
 
 @pytest.mark.parametrize("nb", [300, 700, 1100, 2100])
 def test_inverse_general_tall_panels(ctx, nb):
-    """Every pivot search variant (rows per thread, threads), on a matrix whose pivots lie far from
-    the diagonal and with equal candidates (a permuted diagonal of equal entries).  The residual of
+    """The pivot searches with a panel's rows in registers (rows per thread, threads), on a matrix
+    whose pivots lie far from the diagonal and with equal candidates (a permuted diagonal of equal entries).  The residual of
     A inv(A) is bounded by nb cond(A) 2^-53 times 8 for an elimination without growth."""
     g = np.random.default_rng(nb)
     A = (g.standard_normal((nb, nb)) + 1j * g.standard_normal((nb, nb))) / (4 * np.sqrt(nb))
@@ -291,3 +291,20 @@ def test_inverse_general_tall_panels(ctx, nb):
     d.free()
     s = np.linalg.svd(A, compute_uv=False)
     assert np.abs(A @ X - np.eye(nb)).max() < 8 * nb * (s[0] / s[-1]) * 2.0**-53
+
+
+@pytest.mark.parametrize("nb", [2400, 4100])
+def test_inverse_general_largest_panels(ctx, nb):
+    """Above 2304 rows the columns are put back two rows at a time; above 4096 the pivots are
+    applied one by one in memory.  4 P + G with a permutation P and a random G of norm 0.7 has
+    condition 1.5; the residual of A inv(A) is bounded by nb cond(A) 2^-53 times 8."""
+    g = np.random.default_rng(nb)
+    A = (g.standard_normal((nb, nb)) + 1j * g.standard_normal((nb, nb))) / (4 * np.sqrt(nb))
+    A[np.arange(nb), g.permutation(nb)] += 4.0
+    d = ctx.to_dev(np.ascontiguousarray(A.T))
+    ctx.inverse_general_dev(d, nb, 1, nb)
+    X = d.download(np.complex128, (nb, nb)).T
+    d.free()
+    r = A @ X
+    r[np.diag_indices(nb)] -= 1.0
+    assert np.abs(r).max() < 8 * nb * 1.5 * 2.0**-53
