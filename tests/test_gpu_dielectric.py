@@ -142,9 +142,10 @@ def _eliminate(a):
 def test_hpd_inverse_keeps_the_eliminations_accuracy(ctx, nb, cond):
     """eps = 1 + V B B^H V with a dense v^1/2 of condition 1e3: the leading 16 x 16 blocks are as
     ill conditioned as the matrix.  The blocked inverse performs the operations of the elimination
-    pivot by pivot, rounded in another association, so its error (geometric mean over eight
-    matrices, against extended precision) is of the same size; 2 is asked for.  Products with
-    explicit inverses of the 16 x 16 blocks reach 7 to 7000."""
+    pivot by pivot in their order, so its error (geometric mean over eight matrices, against
+    extended precision) is the same up to the rounding of single products; 1.1 times it is asked
+    for (measured 0.94 to 1.04).  Products with explicit inverses of the 16 x 16 blocks reach 7 to
+    7000 times it."""
     g = np.random.default_rng(nb)
     cn = lambda *s: g.standard_normal(s) + 1j * g.standard_normal(s)
     A = []
@@ -166,7 +167,7 @@ def test_hpd_inverse_keeps_the_eliminations_accuracy(ctx, nb, cond):
                     for y in (x, _eliminate(a))])
     e, ref = np.exp(np.mean(np.log(err), axis=0))
     print(f"nb={nb} cond={cond:.0e}: {e:.2e}, pivot by pivot {ref:.2e}")
-    assert e < 2 * ref, (e, ref)
+    assert e < 1.1 * ref, (e, ref)
 
 
 class _Off:
