@@ -333,7 +333,9 @@ int spexhip_chi0_cplx_dev(spexhip_ctx *ctx, long n, int nb, const void *M_dev, l
 /* One q-point's pair sum (susceptibility.f:1159-1251) as a problem of a
  * grouped launch: M_dev transition-major (t*ldm + I), wght_dev (n x nw, t
  * fastest), chi_dev full column-major per frequency;
- * chi = beta*chi + alpha*sum_t w M conj(M).                               */
+ * chi = beta*chi + alpha*sum_t w M conj(M).  A grouped launch sums every
+ * tile whole, spexhip_chi0_dev in parts where tiles are few: the two agree
+ * to rounding.                                                            */
 typedef struct {
   long n;
   int nb, nw;

@@ -970,13 +970,14 @@ int spx_pw_plan_build(spexhip_ctx *ctx, const spexhip_pw_desc *d, spexhip_plan *
   // the exact convolution -- the same numbers on every such grid, the
   // caller's included.  The plan then uses the smallest such grid (at least
   // the 16-point box); a caller grid that aliases is kept as given.
-  // Sizes are rounded up to 16, 20, 24 or 32 (the in-plane sizes with a
-  // specialised pair kernel) when that is still below the caller's grid.
+  // The box holds W <= 15, so that is 24 at most.  Sizes are rounded up to 16,
+  // 20 or 24 where that is still below the caller's grid (18 and 21 have square
+  // kernels too, but have not been timed against 20 and 24).
   const bool theta = d->step_r || d->step_c;
   if (!theta)
     for (int i = 0; i < 3; i++) {
       int nmin = std::max(PW_BOX, hi[i] >= lo[i] ? hi[i] - lo[i] + PW_OFF + 1 : PW_BOX);
-      for (int nice : {16, 20, 24, 32})
+      for (int nice : {16, 20, 24})
         if (nmin <= nice && nice <= p->nfft[i]) {
           nmin = nice;
           break;
