@@ -41,6 +41,24 @@ def _run(ctx, nkpt3, rl, eo, eu, frq, efermi=0.0):
             b.free()
 
 
+@pytest.mark.parametrize("nunocc", [1, 7, 70])
+@pytest.mark.parametrize("ef", [0.0, 0.2])
+def test_tetra_weights_do_not_depend_on_the_order_of_bands(ctx, nunocc, ef):
+    """Each transition's weights depend on its own energies only, whether the lanes of its wave walk
+    their own bins (bands far apart) or the wave's together (bands alike): permuting the bands
+    permutes the weights bit for bit, for an insulator and with bands that the Fermi energy cuts."""
+    g = np.random.default_rng(nunocc)
+    nk3, frq = (3, 2, 3), 0.03 * (1.05 ** np.arange(50) - 1)
+    eo = -g.uniform(0.05, 0.3, (18, 3)) + ef
+    # alternating groups: wide random bands, and narrow ones at different heights
+    eu = g.uniform(0.05, 0.4, (18, nunocc)) + np.where(np.arange(nunocc) // 20 % 2, 0.0, 0.02 * np.arange(nunocc))
+    ref = _run(ctx, nk3, RL_SKEW, eo, eu, frq, efermi=ef).reshape(18, 3, nunocc, -1)
+    for seed in range(3):
+        p = np.random.default_rng(seed).permutation(nunocc)
+        got = _run(ctx, nk3, RL_SKEW, eo, np.ascontiguousarray(eu[:, p]), frq, efermi=ef)
+        np.testing.assert_array_equal(got.reshape(18, 3, nunocc, -1), ref[:, :, p])
+
+
 @pytest.mark.parametrize("nkpt3,rl,frq0", [
     ((3, 2, 2), np.eye(3), 0.0),
     ((2, 3, 3), RL_SKEW, 0.02),
