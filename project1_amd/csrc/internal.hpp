@@ -28,7 +28,7 @@ size_t spx_wfprod_pw_ws_core(const spexhip_plan *p, int nocc, int nunocc);
 int spx_wfprod_pw_async(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p, const void *cpw,
                         int nband, int nk, const int *k1, const int *k2, const int *oidx_dev,
                         int b1lo, int nocc, int b2lo, int nunocc, void *M, long ldm, int col0,
-                        void *ws);
+                        void *ws, size_t ws_bytes = 0);
 // dielectric step and inverse
 int spx_dielectric(spexhip_ctx *ctx, hipStream_t st, int nb, int nw, void *X, long ldx, int vkind,
                    const void *vh, void *E, long lde, void *tmp);

@@ -16,8 +16,8 @@ int spx_wfprod_mt(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p, const
 size_t spx_wfprod_mt_ws(const spexhip_plan *p, int nk, int nocc, int nunocc);
 int spx_wfprod_pw(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p, const void *cpw,
                   int nband, int nk, const int *k1, const int *k2, const int *g2, int b1lo,
-                  int nocc, int b2lo, int nunocc, void *M, long ldm, int col0, void *ws);
-size_t spx_wfprod_pw_ws(const spexhip_plan *p, int nk, int nocc, int nunocc);
+                  int nocc, int b2lo, int nunocc, void *M, long ldm, int col0, void *ws, bool two);
+size_t spx_wfprod_pw_ws(const spexhip_plan *p, int nk, int nocc, int nunocc, bool two);
 int spx_transpose_d2h(spexhip_ctx *ctx, hipStream_t st, const void *M, long rows, int cols,
                       long ldm, double *host_colmajor);
 
@@ -144,10 +144,13 @@ int spexhip_wfprod2_pw_dev(spexhip_ctx *ctx, const spexhip_plan *plan, const voi
             "wfprod_pw: cpw is not a context allocation of maxgpt*nband*nkpt complex");
   SPX_HIP(ctx, hipSetDevice(ctx->device));
   void *ws;
-  rc = spx_scratch(ctx, spx_wfprod_pw_ws(plan, nk, nocc, nunocc), &ws);
+  bool two = true;  // k points at a time, if the budget has room
+  rc = spx_scratch(ctx, spx_wfprod_pw_ws(plan, nk, nocc, nunocc, two), &ws);
+  if (rc == SPEXHIP_E_NOMEM)
+    rc = spx_scratch(ctx, spx_wfprod_pw_ws(plan, nk, nocc, nunocc, two = false), &ws);
   if (rc) return rc;
   return spx_wfprod_pw(ctx, ctx->stream, plan, cpw_dev, nband, nk, k1, k2, g2, b1lo, nocc, b2lo,
-                       nunocc, M_dev, ldm, col0, ws);
+                       nunocc, M_dev, ldm, col0, ws, two);
 }
 
 int spexhip_wavefproducts2_mt(spexhip_ctx *ctx, const spexhip_plan *plan, const double *cmt,

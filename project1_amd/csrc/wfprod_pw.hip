@@ -1003,8 +1003,18 @@ int spx_pw_plan_build(spexhip_ctx *ctx, const spexhip_pw_desc *d, spexhip_plan *
 }
 
 size_t spx_wfprod_pw_ws_core(const spexhip_plan *p, int nocc, int nunocc);
-size_t spx_wfprod_pw_ws(const spexhip_plan *p, int nk, int nocc, int nunocc) {
-  return spx_wfprod_pw_ws_core(p, nocc, nunocc) + 4 * (size_t)nk * p->ngptm + 256;
+// Workspace of the synchronous form: grids, then the oidx table.  two: room for
+// two k points' grids on square planes where the core has room for two in the
+// natural layout but not in the square one's (up to a quarter larger): one k
+// point at a time of 8 x 56 states on 36^3 points, 112 workgroups, takes 1.95 ms
+// for eight of them, two together 0.99.
+static size_t pw_grid_bytes(const spexhip_plan *p, int nocc, int nunocc, bool two) {
+  const size_t core = spx_wfprod_pw_ws_core(p, nocc, nunocc), set = square_set(p, nocc, nunocc);
+  const size_t plain = 16 * (size_t)(nocc + nunocc) * p->nfft[0] * p->nfft[1] * p->nfft[2];
+  return two && set && core >= 2 * plain ? std::max(core, 2 * set) : core;
+}
+size_t spx_wfprod_pw_ws(const spexhip_plan *p, int nk, int nocc, int nunocc, bool two) {
+  return pw_grid_bytes(p, nocc, nunocc, two && nk > 1) + 4 * (size_t)nk * p->ngptm + 256;
 }
 
 // Box indices of imati.(Gm - g2(k)) for every packet k and IPW (host).
@@ -1031,16 +1041,17 @@ size_t spx_wfprod_pw_ws_core(const spexhip_plan *p, int nocc, int nunocc) {
 }
 
 // Asynchronous launches (no host synchronisation): k1, k2 are host arrays
-// used as launch arguments, oidx_dev a device table from spx_pw_oidx.
+// used as launch arguments, oidx_dev a device table from spx_pw_oidx.  ws_bytes:
+// of ws where it holds more than the core.
 int spx_wfprod_pw_async(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p, const void *cpw,
                         int nband, int nk, const int *k1, const int *k2, const int *oidx_dev,
                         int b1lo, int nocc, int b2lo, int nunocc, void *M, long ldm, int col0,
-                        void *ws) {
+                        void *ws, size_t ws_bytes) {
   for (int ik = 0; ik < nk; ik++)
     SPX_CHECK(ctx, k1[ik] >= 0 && k1[ik] < p->nkpt && k2[ik] >= 0 && k2[ik] < p->nkpt,
               "wfprod_pw: k index out of range");
   if (const size_t set = square_set(p, nocc, nunocc)) {
-    const size_t fit = spx_wfprod_pw_ws_core(p, nocc, nunocc) / set;
+    const size_t fit = std::max(ws_bytes, spx_wfprod_pw_ws_core(p, nocc, nunocc)) / set;
     return launch_square(ctx, st, p, cpw, nband, nk, k1, k2, oidx_dev, b1lo, nocc, b2lo, nunocc, M,
                          ldm, col0, ws, (int)std::min<size_t>(fit, PW_KMAX));
   }
@@ -1059,14 +1070,15 @@ int spx_wfprod_pw_async(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p,
 // Synchronous form: builds and uploads the oidx table into the tail of ws.
 int spx_wfprod_pw(spexhip_ctx *ctx, hipStream_t st, const spexhip_plan *p, const void *cpw,
                   int nband, int nk, const int *k1, const int *k2, const int *g2, int b1lo,
-                  int nocc, int b2lo, int nunocc, void *M, long ldm, int col0, void *ws) {
+                  int nocc, int b2lo, int nunocc, void *M, long ldm, int col0, void *ws, bool two) {
+  const size_t gb = pw_grid_bytes(p, nocc, nunocc, two && nk > 1);
   std::vector<int> oidx((size_t)nk * p->ngptm);
   int rc = spx_pw_oidx(ctx, p, nk, g2, oidx.data());
   if (rc) return rc;
-  int *oidx_dev = (int *)((char *)ws + spx_wfprod_pw_ws_core(p, nocc, nunocc));
+  int *oidx_dev = (int *)((char *)ws + gb);
   SPX_HIP(ctx, hipMemcpyAsync(oidx_dev, oidx.data(), 4 * oidx.size(), hipMemcpyHostToDevice, st));
   rc = spx_wfprod_pw_async(ctx, st, p, cpw, nband, nk, k1, k2, oidx_dev, b1lo, nocc, b2lo, nunocc,
-                           M, ldm, col0, ws);
+                           M, ldm, col0, ws, gb);
   SPX_HIP(ctx, hipStreamSynchronize(st));  // oidx is a host temporary
   return rc;
 }

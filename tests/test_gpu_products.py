@@ -322,3 +322,24 @@ def test_pw_skewed_lattice_complex_step_grid(ctx):
     mx, fro = normwise(got, ref)
     print(f"PW skewed basis, complex theta nfft={nfft}: max-rel {mx:.2e} fro-rel {fro:.2e}")
     assert mx < TOL
+
+
+def test_pw_two_k_points_where_the_grids_fit_twice(ctx):
+    """8 x 56 states on 36^3 points: the workspace holds two k points' grids in the natural layout
+    but not in the square planes' one, so a call of several k points takes a little more; without
+    room for it (a context budget) one k point at a time gives the same bits."""
+    s = synth.product_system(nmesh=2, nband=64, gcut=3.1, gcutm=2.1, nfft=(36, 36, 36), seed=61)
+    th = np.random.default_rng(1).uniform(0.5, 1.0, 36**3)
+    nset = 64 * 18 * 25 * 128 * 16  # bytes of one k point's grids
+    core = 16 * (64 * 36**3 + 8 * 56 * 36 * 256)
+    assert nset < core < 2 * nset
+    with spexhip.Context(0) as c:
+        want = _pw_dev(c, s, 0, 8, 8, 56, step=th)
+        used = c.mem_used()[0]  # the scratch
+        one = _pw_dev(c, synth.ProductSystem(**{**s.__dict__, "k1": s.k1[3:4], "k2": s.k2[3:4],
+                                                "g2": s.g2[3:4]}), 0, 8, 8, 56, step=th)
+    np.testing.assert_array_equal(one, want[3 * 448:4 * 448])
+    assert used >= 2 * nset
+    with spexhip.Context(0, hbm_budget=used - (1 << 20)) as c:
+        np.testing.assert_array_equal(_pw_dev(c, s, 0, 8, 8, 56, step=th), want)
+        assert c.mem_used()[0] < used
