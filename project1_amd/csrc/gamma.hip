@@ -212,7 +212,7 @@ __global__ __launch_bounds__(HW_NT) void headwing_kernel(
 // weights too, 12 streams a wave thrash the scalar cache: 4.6 ms).  Staging M
 // in LDS as for column-major M leaves room for one wave per SIMD only.
 // 409,600 transitions x 1200 columns x 12 frequencies: 2.6 -> 1.96 ms, VALU
-// busy 72 %: bound by the 84 FP64 FMAs per entry of M at the 1.9 GHz that the
+// busy 70 %: bound by the 84 FP64 FMAs per entry of M at the 1.9 GHz that the
 // card then runs at, beside reading M at 4 TB/s.
 template <bool CPLX, int NWB>
 __global__ __launch_bounds__(HW_NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
