@@ -41,7 +41,8 @@ enum {
 
 enum {
   SPEXHIP_PREC_FP64 = 0,       /* plain FP64 MFMA                          */
-  SPEXHIP_PREC_SPLIT_FP32 = 1, /* hi+lo FP32 operands, 3 FP32 MFMA products,
+  SPEXHIP_PREC_SPLIT_FP32 = 1, /* integer hi + FP32 lo operands: hi*hi on FP16
+                                  MFMA (exact), the rest in FP32 products,
                                   FP32 accumulation in short K-chunks flushed
                                   into FP64 accumulators                     */
   SPEXHIP_PREC_OZAKI_INT8 = 2  /* weights balanced as sqrt|D| on both sides,
